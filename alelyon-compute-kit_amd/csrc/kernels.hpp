@@ -40,7 +40,8 @@ enum class MatmulPath : int {
   GemvDirect = 7,    // m <= 8, few weights (kDirectMaxWeights): decode and FMA per output,
                      // split k reduced by the last block of each tile, one launch
   OneHotMfma = 8,    // m >= kOneHotMinRows, packed A along k, B along n: A's book rows x
-                     // one-hot of B's codes on bf16 MFMA, then the 16-term codebook product
+                     // one-hot of B's codes on bf16 MFMA (six-bit digits on large grids),
+                     // then the 16-term codebook product
   GeneralMfma = 10,  // General's shapes from kGeneralMinMacs: both operands decoded into bf16
                      // terms, six MFMA products (also named "general")
   JointMfma = 9,     // A stored k x m, both grouped along the output's sides: pair counts of
