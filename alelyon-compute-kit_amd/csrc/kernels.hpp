@@ -66,7 +66,9 @@ hipError_t launch_sum_squares(hipStream_t s, const float* x, uint64_t count, dou
                               double* out);
 // x[i] *= f in FP32, in place.
 hipError_t launch_scale(hipStream_t s, float* x, uint64_t count, float f);
-// the k slices' partial sums on small grids; without a workspace one slice runs
+// The k slices' partial sums of the gram and general paths on small grids (0 where
+// blocks walk the slices); without a workspace they are walked too, with the same bits.
+constexpr size_t kBatchPartialBytes = size_t(64) << 20;
 size_t gram_workspace_bytes(uint32_t m, uint32_t n, uint32_t k, uint32_t group, uint32_t count);
 hipError_t launch_gram(hipStream_t s, const Operands& o, uint32_t m, uint32_t n, uint32_t k,
                        uint32_t group, void* workspace);
@@ -138,8 +140,9 @@ constexpr uint32_t kJointMinK = 12, kJointMinK8 = 48;
 constexpr uint64_t kJointMinMacs = 1ull << 22;
 constexpr size_t kJointMaxWorkspace = size_t(256) << 20;
 bool joint_applies(uint32_t m, uint32_t n, uint32_t k, uint32_t group, uint32_t flags,
-                   uint32_t count, bool any_size);
-// the transposed codes of both operands, `count` times
+                   bool any_size);
+// the transposed codes of both operands, `count` times, up to kJointMaxWorkspace;
+// without them (0, or no workspace) the blocks transpose their own
 size_t joint_workspace_bytes(uint32_t m, uint32_t n, uint32_t k, uint32_t group, uint32_t count);
 hipError_t launch_joint(hipStream_t s, const Operands& o, uint32_t m, uint32_t n, uint32_t k,
                         uint32_t group, void* workspace);

@@ -25,9 +25,11 @@
 // 250 KB per 128 x 128 x 32 stage against 1,540 matrix cycles a wave) on large
 // products, the loads' latency and the second launch on small ones.
 //
-// Grids of fewer than kGeneralBlocks blocks cut k into slices; the slices'
-// sums go to the workspace (at most 8 MiB) and k_sum_slices adds them in
-// slice order.
+// Grids of fewer than kGeneralBlocks blocks cut k into slices. They run side by
+// side, their sums go to the workspace and k_sum_slices adds them in slice order;
+// or, in batches that fill the chip and where there is no workspace, each block
+// walks the slices and adds their sums in the same order in the output. The slices
+// are those of the product alone, so neither changes a bit.
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
@@ -48,7 +50,7 @@ constexpr uint32_t kStageK = 32;       // inner indices per stage
 constexpr uint32_t kChunks = kStageK / 8;
 constexpr int kTerms = 3;
 constexpr uint32_t kGeneralBlocks = 512;
-constexpr uint64_t kPartialBytes = uint64_t(8) << 20;
+constexpr uint64_t kPartialBytes = uint64_t(8) << 20;  // of one product's slices
 
 // How an operand of R rows (A) or columns (B) lies in memory.
 enum Source : int {
@@ -270,9 +272,10 @@ struct Loader {
   }
 };
 
-// grid: (ceil(n / 128), ceil(m / BM), instances * slices). The block's 4 waves
-// lie 2 x 2 (BM 64 and 128) or 1 x 4 (BM 32) over the tile.
-template <int ASRC, int BSRC, uint32_t BM>
+// grid: (ceil(n / 128), ceil(m / BM), instances * slices, or instances where the
+// blocks walk the slices: WALK). The block's 4 waves lie 2 x 2 (BM 64
+// and 128) or 1 x 4 (BM 32) over the tile.
+template <int ASRC, int BSRC, uint32_t BM, bool WALK>
 __global__ __launch_bounds__(kThreads, 2) void k_general_mfma(Operands o, uint32_t m, uint32_t n,
                                                               uint32_t k, uint32_t lg,
                                                               uint32_t slices, uint32_t slice_k,
@@ -289,13 +292,15 @@ __global__ __launch_bounds__(kThreads, 2) void k_general_mfma(Operands o, uint32
   const uint32_t wr = wave / (4 / kWaveRows) * (32 * X), wc = wave % (4 / kWaveRows) * (32 * Y);
   const uint32_t entries = 16u << lg;
 
-  for (uint32_t z = blockIdx.z; z < o.count * slices; z += gridDim.z) {
-    const uint32_t item = z / slices, slice = z % slices;
+  const uint32_t each = WALK ? slices : 1;  // slices of a block
+  for (uint32_t z = blockIdx.z * each; z < o.count * slices; z += gridDim.z * each) {
+    const uint32_t item = z / slices;
+    uint32_t slice = z % slices;
     const void* a = item_ptr<char>(o.in[0], o.stride[0], item);
     const float* a_book = item_ptr<float>(o.in[1], o.stride[1], item);
     const void* b = item_ptr<char>(o.in[2], o.stride[2], item);
     const float* b_book = item_ptr<float>(o.in[3], o.stride[3], item);
-    const uint32_t kbeg = slice * slice_k, kend = k - kbeg < slice_k ? k : kbeg + slice_k;
+    uint32_t kbeg = slice * slice_k, kend = k - kbeg < slice_k ? k : kbeg + slice_k;
 
     // loads run kAhead stages ahead; the 128-row tile has no registers for two
     constexpr uint32_t kAhead = BM == 128 ? 1 : 2;
@@ -326,10 +331,6 @@ __global__ __launch_bounds__(kThreads, 2) void k_general_mfma(Operands o, uint32
     if constexpr (!kDenseA) fill_table(ta, a_book, entries, shift.a);
     fill_table(tb, b_book, entries, shift.b);
     f32x16 acc[X][Y];
-#pragma unroll
-    for (uint32_t x = 0; x < X; ++x)
-#pragma unroll
-      for (uint32_t y = 0; y < Y; ++y) acc[x][y] = (f32x16)0.0f;
     __syncthreads();
 
     auto step = [&](Loader<ASRC, BM>& x, Loader<BSRC, kTileN>& y, uint32_t k0) {
@@ -368,31 +369,46 @@ __global__ __launch_bounds__(kThreads, 2) void k_general_mfma(Operands o, uint32
       }
       __syncthreads();
     };
-    for (uint32_t k0 = kbeg; k0 < kend; k0 += kAhead * kStageK)
-#pragma unroll
-      for (uint32_t x = 0; x < kAhead; ++x)
-        if (k0 + x * kStageK < kend) step(la[x], lb[x], k0 + x * kStageK);
-
-    float* out = reinterpret_cast<float*>(static_cast<char*>(o.out) + o.stride[4] * item);
-    const bool direct = slices == 1;
-    if (!direct) out = partial + uint64_t(z) * m * n;
+    const bool direct = WALK || slices == 1;
+    float* out = direct ? reinterpret_cast<float*>(static_cast<char*>(o.out) + o.stride[4] * item)
+                        : partial + uint64_t(z) * m * n;
     const int up = -(shift.a + shift.b);
-    uint32_t rows = m, columns = n;  // as above: not 64 bounds tests kept over the loop
-    asm volatile("" : "+s"(rows), "+s"(columns));
+    for (uint32_t left = each;;) {
 #pragma unroll
-    for (uint32_t x = 0; x < X; ++x)
+      for (uint32_t x = 0; x < X; ++x)
 #pragma unroll
-      for (uint32_t y = 0; y < Y; ++y)
+        for (uint32_t y = 0; y < Y; ++y) acc[x][y] = (f32x16)0.0f;
+      for (uint32_t k0 = kbeg; k0 < kend; k0 += kAhead * kStageK)
 #pragma unroll
-        for (uint32_t t = 0; t < 16; ++t) {
-          const uint32_t r = m0 + wr + 32 * x + (t % 4) + 4 * h + 8 * (t / 4);
-          const uint32_t c = n0 + wc + 32 * y + i32;
-          if (r < rows && c < columns) {
-            const float v = ldexpf(acc[x][y][t], up);
-            out[uint64_t(r) * columns + c] = v;
-            bad |= direct && !finite_f32(v);
+        for (uint32_t x = 0; x < kAhead; ++x)
+          if (k0 + x * kStageK < kend) step(la[x], lb[x], k0 + x * kStageK);
+
+      uint32_t rows = m, columns = n;  // as above: not 64 bounds tests kept over the loop
+      asm volatile("" : "+s"(rows), "+s"(columns));
+      const bool last = direct && (!WALK || left == 1);
+#pragma unroll
+      for (uint32_t x = 0; x < X; ++x)
+#pragma unroll
+        for (uint32_t y = 0; y < Y; ++y)
+#pragma unroll
+          for (uint32_t t = 0; t < 16; ++t) {
+            const uint32_t r = m0 + wr + 32 * x + (t % 4) + 4 * h + 8 * (t / 4);
+            const uint32_t c = n0 + wc + 32 * y + i32;
+            if (r < rows && c < columns) {
+              float* at = out + uint64_t(r) * columns + c;
+              float v = ldexpf(acc[x][y][t], up);
+              if (WALK) v = (slice > 0 ? *at : 0.0f) + v;
+              *at = v;
+              bad |= last && !finite_f32(v);
+            }
           }
-        }
+      if (!WALK || --left == 0) break;
+      ++slice;
+      kbeg = kend;
+      kend = k - kbeg < slice_k ? k : kbeg + slice_k;
+#pragma unroll
+      for (uint32_t x = 0; x < kAhead; ++x) load(la[x], lb[x], kbeg + x * kStageK);
+    }
     if (__any(bad) && lane == 0) atomicOr(o.status, 1u);
   }
 }
@@ -425,17 +441,19 @@ struct GeneralGrid {
   uint32_t bm, gx, gy, slices, slice_k;
 };
 
-// 128-row blocks where they (times their slices) fill the chip, else 64-row
-// ones, 32 for fewer rows.
+// The slices of one product, whatever batch it is in: 128-row blocks where they
+// (times their slices) fill the chip, else 64-row ones, 32 for fewer rows. In a
+// batch the blocks may be larger, which changes no sum.
 GeneralGrid general_grid(uint32_t m, uint32_t n, uint32_t k, uint32_t count) {
   const uint64_t stages = (k + kStageK - 1) / kStageK;
-  const uint64_t room = kPartialBytes / (uint64_t(m) * n * 4 * count);
+  const uint64_t room = kPartialBytes / (uint64_t(m) * n * 4);
+  const uint32_t most = m <= 32 ? 32 : m <= 64 ? 64 : 128;
   GeneralGrid g;
   uint64_t slices = 1;
-  for (g.bm = m <= 32 ? 32 : m <= 64 ? 64 : 128;; g.bm = 64) {
-    g.gx = (n + kTileN - 1) / kTileN;
+  g.gx = (n + kTileN - 1) / kTileN;
+  for (g.bm = most;; g.bm = 64) {
     g.gy = (m + g.bm - 1) / g.bm;
-    const uint64_t blocks = uint64_t(g.gx) * g.gy * count;
+    const uint64_t blocks = uint64_t(g.gx) * g.gy;
     slices = (kGeneralBlocks + blocks - 1) / blocks;
     if (slices > room) slices = room;
     if (slices > stages / 2) slices = stages / 2;
@@ -444,20 +462,33 @@ GeneralGrid general_grid(uint32_t m, uint32_t n, uint32_t k, uint32_t count) {
   }
   g.slice_k = uint32_t((stages + slices - 1) / slices) * kStageK;
   g.slices = (k + g.slice_k - 1) / g.slice_k;
+  if (g.bm < most && uint64_t(g.gx) * ((m + most - 1) / most) * count >= kGeneralBlocks / 2) {
+    g.bm = most;
+    g.gy = (m + most - 1) / most;
+  }
   return g;
+}
+
+template <int ASRC, int BSRC, uint32_t BM>
+void run_general_rows(hipStream_t s, const Operands& o, uint32_t m, uint32_t n, uint32_t k,
+                      uint32_t lg, const GeneralGrid& g, float* partial) {
+  const bool walk = partial == nullptr && g.slices > 1;
+  const uint64_t z = uint64_t(o.count) * (walk ? 1 : g.slices);
+  const dim3 grid(g.gx, g.gy, z < 65535 ? uint32_t(z) : 65535u);
+  if (walk)
+    k_general_mfma<ASRC, BSRC, BM, true><<<grid, kThreads, 0, s>>>(o, m, n, k, lg, g.slices,
+                                                                   g.slice_k, partial);
+  else
+    k_general_mfma<ASRC, BSRC, BM, false><<<grid, kThreads, 0, s>>>(o, m, n, k, lg, g.slices,
+                                                                    g.slice_k, partial);
 }
 
 template <int ASRC, int BSRC>
 void run_general(hipStream_t s, const Operands& o, uint32_t m, uint32_t n, uint32_t k, uint32_t lg,
                  const GeneralGrid& g, float* partial) {
-  const uint64_t z = uint64_t(o.count) * g.slices;
-  const dim3 grid(g.gx, g.gy, z < 65535 ? uint32_t(z) : 65535u);
-  if (g.bm == 32)
-    k_general_mfma<ASRC, BSRC, 32><<<grid, kThreads, 0, s>>>(o, m, n, k, lg, g.slices, g.slice_k, partial);
-  else if (g.bm == 64)
-    k_general_mfma<ASRC, BSRC, 64><<<grid, kThreads, 0, s>>>(o, m, n, k, lg, g.slices, g.slice_k, partial);
-  else
-    k_general_mfma<ASRC, BSRC, 128><<<grid, kThreads, 0, s>>>(o, m, n, k, lg, g.slices, g.slice_k, partial);
+  if (g.bm == 32) run_general_rows<ASRC, BSRC, 32>(s, o, m, n, k, lg, g, partial);
+  else if (g.bm == 64) run_general_rows<ASRC, BSRC, 64>(s, o, m, n, k, lg, g, partial);
+  else run_general_rows<ASRC, BSRC, 128>(s, o, m, n, k, lg, g, partial);
 }
 
 template <int ASRC>
@@ -477,14 +508,18 @@ void launch_sum_slices(hipStream_t s, const Operands& o, uint32_t mn, uint32_t s
 
 size_t general_workspace_bytes(uint32_t m, uint32_t n, uint32_t k, uint32_t count) {
   const GeneralGrid g = general_grid(m, n, k, count);
-  return g.slices == 1 ? 0 : size_t(m) * n * 4 * count * g.slices;
+  const size_t bytes = size_t(m) * n * 4 * count * g.slices;
+  const bool walk = g.slices == 1 || uint64_t(g.gx) * g.gy * count >= kGeneralBlocks ||
+                    bytes > kBatchPartialBytes;
+  return walk ? 0 : bytes;
 }
 
 hipError_t launch_general_mfma(hipStream_t s, const Operands& o, uint32_t m, uint32_t n, uint32_t k,
                                uint32_t group, uint32_t flags, bool dense, void* workspace) {
   const GeneralGrid g = general_grid(m, n, k, o.count);
   const uint32_t lg = group == 8 ? 3 : group == 16 ? 4 : 5;
-  float* partial = static_cast<float*>(workspace);
+  float* partial =
+      general_workspace_bytes(m, n, k, o.count) == 0 ? nullptr : static_cast<float*>(workspace);
   if (dense) {
     if (flags & 1u) run_general_b<kDenseAlongR>(s, o, m, n, k, lg, flags, g, partial);
     else run_general_b<kDenseAlongK>(s, o, m, n, k, lg, flags, g, partial);
@@ -492,7 +527,7 @@ hipError_t launch_general_mfma(hipStream_t s, const Operands& o, uint32_t m, uin
     if (flags & 1u) run_general_b<kPackedAlongR>(s, o, m, n, k, lg, flags, g, partial);
     else run_general_b<kPackedAlongK>(s, o, m, n, k, lg, flags, g, partial);
   }
-  if (g.slices > 1) launch_sum_slices(s, o, m * n, g.slices, partial);
+  if (partial != nullptr) launch_sum_slices(s, o, m * n, g.slices, partial);
   return hipGetLastError();
 }
 

@@ -54,7 +54,8 @@ constexpr uint32_t kJointStep = 128;     // inner indices per MFMA
 // Up to this k the blocks transpose their own codes: the pre-pass's launch and
 // its ~4 us outweigh the repeated reads (4096 x 4096 at group 16: k = 32 19.4
 // against 22.3 us, 256 22.5 against 23.8, 512 27.8 against 26.7; 4096 x 14336,
-// k = 2048 185 against 131).
+// k = 2048 185 against 131). So they do without a workspace for the transposed
+// codes; the counts are whole numbers, so the outputs have the same bits.
 constexpr uint32_t kJointGather = 256;
 constexpr int kFp4 = 4;                  // the instruction's code for e2m1 operands
 
@@ -384,24 +385,24 @@ void choose_joint(hipStream_t s, const Operands& o, uint32_t m, uint32_t n, uint
 }  // namespace
 
 bool joint_applies(uint32_t m, uint32_t n, uint32_t k, uint32_t group, uint32_t flags,
-                   uint32_t count, bool any_size) {
+                   bool any_size) {
   if (flags != 1 || m % group != 0 || n % group != 0 || m < kJointMinRows) return false;
   if (!any_size && k < (group == 8 ? kJointMinK8 : kJointMinK)) return false;
-  if (joint_workspace_bytes(m, n, k, group, count) > kJointMaxWorkspace) return false;
-  return any_size || uint64_t(m) * n * k * count >= kJointMinMacs;
+  return any_size || uint64_t(m) * n * k >= kJointMinMacs;
 }
 
 size_t joint_workspace_bytes(uint32_t m, uint32_t n, uint32_t k, uint32_t group, uint32_t count) {
   if (k <= kJointGather) return 0;
-  return size_t(m / group + n / group) * (padded_k(k) / 8) * 4 * count;
+  const size_t bytes = size_t(m / group + n / group) * (padded_k(k) / 8) * 4 * count;
+  return bytes <= kJointMaxWorkspace ? bytes : 0;
 }
 
 hipError_t launch_joint(hipStream_t s, const Operands& o, uint32_t m, uint32_t n, uint32_t k,
                         uint32_t group, void* workspace) {
   const uint32_t z = o.count < 65535 ? o.count : 65535;
-  uint32_t* words = nullptr;
-  if (k > kJointGather) {
-    words = static_cast<uint32_t*>(workspace);
+  uint32_t* words = joint_workspace_bytes(m, n, k, group, o.count) == 0
+                        ? nullptr : static_cast<uint32_t*>(workspace);
+  if (words != nullptr) {
     const uint32_t va = m / group, vb = n / group;
     const dim3 pre((va + vb + 63) / 64, (padded_k(k) / 32 + 3) / 4, z);
     k_joint_words<<<pre, 256, 0, s>>>(o, va, vb, k, words);

@@ -1917,11 +1917,11 @@ const char* matmul_path_name(MatmulPath p) {
   return "unknown";
 }
 
-// What serves the shapes no factorised path takes.
-static MatmulPath general_path(uint32_t m, uint32_t n, uint32_t k, uint32_t count,
-                               uint32_t policy) {
+// What serves the shapes no factorised path takes: by the product alone, so that
+// it has the same bits in every batch.
+static MatmulPath general_path(uint32_t m, uint32_t n, uint32_t k, uint32_t policy) {
   return policy == 0 && (k >= kGeneralMinK ||
-                         (k >= kGeneralMinKLarge && uint64_t(m) * n * k * count >= kGeneralMinMacs))
+                         (k >= kGeneralMinKLarge && uint64_t(m) * n * k >= kGeneralMinMacs))
              ? MatmulPath::GeneralMfma
              : MatmulPath::General;
 }
@@ -1932,12 +1932,12 @@ MatmulPath choose_matmul_path(uint32_t m, uint32_t n, uint32_t k, uint32_t group
   if ((policy == 0 || m >= kOneHotMinRows) && onehot_applies(m, n, k, group, flags, count))
     return MatmulPath::OneHotMfma;
   if (gram_applies(m, n, k, group, flags, policy == 2)) return MatmulPath::GramMfma;
-  if (joint_applies(m, n, k, group, flags, count, policy == 2)) return MatmulPath::JointMfma;
+  if (joint_applies(m, n, k, group, flags, policy == 2)) return MatmulPath::JointMfma;
   if (policy == 0 && direct_applies(m, n, k, group, flags, count)) return MatmulPath::GemvDirect;
   if (row_pairs_apply(m, n, k, group, flags, count, false)) return MatmulPath::GemvRowPairs;
   if (rows_apply(m, n, k, group, flags))
     return m == 1 ? MatmulPath::GemvPairs : MatmulPath::GemvRows;
-  return general_path(m, n, k, count, policy);
+  return general_path(m, n, k, policy);
 }
 
 size_t matmul_workspace_bytes(MatmulPath p, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
@@ -1998,7 +1998,7 @@ MatmulPath choose_dense_path(uint32_t m, uint32_t n, uint32_t k, uint32_t group,
   if (row_pairs_apply(m, n, k, group, flags, count, true)) return MatmulPath::GemvRowPairs;
   if (rows_apply(m, n, k, group, flags))
     return m == 1 ? MatmulPath::GemvPairs : MatmulPath::GemvRows;
-  return general_path(m, n, k, count, policy);
+  return general_path(m, n, k, policy);
 }
 
 // The factorised paths' split-k partials (the GEMV kernels take each window's
