@@ -42,6 +42,10 @@ struct BufferRec {
   uint64_t id = 0;
 };
 
+// ack_vq_noalloc's area for the workspaces that a path can do without, allocated
+// with the handle: the slices of k of one product fit it.
+constexpr size_t kPartialsBytes = size_t(8) << 20;
+
 struct Device {
   uint64_t id = 0;
   int hip_device = 0;
@@ -58,6 +62,7 @@ struct Device {
   void* workspace = nullptr;
   size_t workspace_bytes = 0;
   void* scratch = nullptr;  // this GPU's copy of `scratch` (ack_vq_noalloc), or null
+  void* partials = nullptr;  // kPartialsBytes for ack_vq_noalloc's optional workspaces, or null
   uint32_t* arrivals = nullptr;  // gemv-direct's counters, zeroed at open (Operands::arrivals)
 };
 
@@ -199,7 +204,10 @@ void* scratch_address(int hip_device) {
   return g_scratch_ptr[hip_device];
 }
 
-int32_t ensure_workspace(Device& dev, size_t bytes) {
+// Grows the handle's workspace to `bytes`. `required` false: a failed allocation
+// leaves no error behind, neither here nor in HIP, whose launches would report it
+// as theirs.
+int32_t ensure_workspace(Device& dev, size_t bytes, bool required = true) {
   if (bytes <= dev.workspace_bytes) return ACK_OK;
   if (dev.workspace) {
     hipError_t e = hipStreamSynchronize(dev.stream);
@@ -210,30 +218,19 @@ int32_t ensure_workspace(Device& dev, size_t bytes) {
   }
   hipError_t e = hipMalloc(&dev.workspace, bytes);
   if (e != hipSuccess) {
+    (void)hipGetLastError();
     dev.workspace = nullptr;
-    return hip_failure(dev, "vq: workspace allocation", e, false);
+    return required ? hip_failure(dev, "vq: workspace allocation", e, false) : ACK_ERR_DEVICE;
   }
   dev.workspace_bytes = bytes;
   return ACK_OK;
 }
 
-// Paths that run without their workspace where it cannot be had: gram-mfma in
-// one slice of k, the others' shapes on the general kernel.
+// Paths that run without their workspace where it cannot be had, slower and with
+// the same bits: blocks walk the slices of k, or gather their own codes.
 bool workspace_optional(ackvq::MatmulPath path) {
   return path == ackvq::MatmulPath::JointMfma || path == ackvq::MatmulPath::GeneralMfma ||
          path == ackvq::MatmulPath::GramMfma;
-}
-
-// Whether ack_vq_noalloc can give this handle `bytes` of its GPU's scratch now.
-bool scratch_free(const Device& dev, size_t bytes) {
-  if (bytes == 0) return true;
-  if (bytes > kScratchBytes || dev.scratch == nullptr) return false;
-  std::lock_guard<std::mutex> lock(g_scratch_mu);
-  const ScratchOwner& own = g_scratch_owner[dev.hip_device];
-  if (own.device == 0 || own.device == dev.id || own.done == nullptr) return true;
-  const hipError_t q = hipEventQuery(own.done);
-  (void)hipGetLastError();  // a pending query must not read as a launch failure
-  return q != hipErrorNotReady;
 }
 
 // Steps 4-7 then the launch, shared by ack_vq, ack_vq_batch and
@@ -302,16 +299,24 @@ int32_t run_vq(const AckDevice* handle, const AckBuffer* const slots[6], const u
       ackvq::MatmulPath path =
           ackvq::choose_matmul_path(m, n, k, g, plan.flags(), count, dev->policy);
       size_t ws = ackvq::matmul_workspace_bytes(path, m, n, k, g, plan.flags(), count);
-      bool no_work = false;
-      if (workspace_optional(path) &&
-          (no_alloc ? !scratch_free(*dev, ws) : ensure_workspace(*dev, ws) != ACK_OK && !dev->poisoned)) {
-        if (path != ackvq::MatmulPath::GramMfma) path = ackvq::MatmulPath::General;
-        no_work = true;
+      // by the plan alone: transposed codes past the scratch's size are not gathered
+      // block by block but left to the shader-order kernel (ack_vq.h)
+      if (no_alloc && path == ackvq::MatmulPath::JointMfma && ws > kScratchBytes) {
+        path = ackvq::MatmulPath::General;
         ws = 0;
       }
       void* work = nullptr;
       size_t work_bytes = 0;
-      if (no_alloc) {
+      if (workspace_optional(path)) {
+        if (no_alloc) {  // the handle's own area: another handle's calls are never in the way
+          if (ws <= kPartialsBytes) work = dev->partials;
+        } else {
+          const int32_t rc = ensure_workspace(*dev, ws, false);
+          if (rc != ACK_OK && dev->poisoned) return rc;
+          if (rc == ACK_OK) work = dev->workspace;
+        }
+        work_bytes = work != nullptr ? ws : 0;
+      } else if (no_alloc) {
         if (ws > kScratchBytes) {
           set_error("vq noalloc: the product needs " + std::to_string(ws) +
                     " bytes of workspace, more than the " + std::to_string(kScratchBytes) +
@@ -357,7 +362,6 @@ int32_t run_vq(const AckDevice* handle, const AckBuffer* const slots[6], const u
         work = dev->workspace;
         work_bytes = dev->workspace_bytes;
       }
-      if (no_work) work = nullptr;
       he = ackvq::launch_matmul(dev->stream, o, m, n, k, g, plan.flags(), path, work, work_bytes);
       break;
     }
@@ -465,6 +469,10 @@ AckDevice* ack_open(void) {
   else
     dev->name = "HIP device " + std::to_string(index);
   if (have_prop) dev->name += std::string(" (") + prop.gcnArchName + ")";
+  if (hipMalloc(&dev->partials, kPartialsBytes) != hipSuccess) {
+    (void)hipGetLastError();
+    dev->partials = nullptr;  // the paths that would use it do without
+  }
   dev->scratch = scratch_address(index);  // `index` is current (hipSetDevice above)
   dev->id = g_next_device.fetch_add(1);
   Registry& r = registry();
@@ -495,12 +503,14 @@ int32_t ack_close(AckDevice* handle) {
                   hipGetErrorString(e));
       if (dev->workspace) (void)hipFree(dev->workspace);
       if (dev->arrivals) (void)hipFree(dev->arrivals);
+      if (dev->partials) (void)hipFree(dev->partials);
       (void)hipEventDestroy(dev->timer_start);
       (void)hipEventDestroy(dev->timer_stop);
       (void)hipStreamDestroy(dev->stream);
     }
     dev->workspace = nullptr;
     dev->arrivals = nullptr;
+    dev->partials = nullptr;
   }
   Registry& r = registry();
   std::lock_guard<std::mutex> lock(r.mu);
@@ -947,12 +957,12 @@ int32_t ack_vq_matmul_dense(const AckDevice* handle, const AckBuffer* x, const A
   for (int i = 0; i < 4; ++i) o.in[i] = bufs[i]->ptr;
   o.out = bufs[4]->ptr;
   o.status = static_cast<uint32_t*>(bufs[5]->ptr);
-  ackvq::MatmulPath path =
+  const ackvq::MatmulPath path =
       ackvq::choose_dense_path(m, n, k, g, plan.flags(), 1, dev->policy);
   const size_t ws = ackvq::dense_workspace_bytes(path, m, n, k, g, plan.flags(), 1);
-  if (int32_t rc = ensure_workspace(*dev, ws)) {
-    if (!workspace_optional(path) || dev->poisoned) return rc;
-    path = ackvq::MatmulPath::General;
+  const bool optional = workspace_optional(path);
+  if (int32_t rc = ensure_workspace(*dev, ws, !optional)) {
+    if (!optional || dev->poisoned) return rc;
   }
   hipError_t he = ackvq::launch_matmul_dense(dev->stream, o, m, n, k, g, plan.flags(), path,
                                              dev->workspace, dev->workspace_bytes);

@@ -217,12 +217,18 @@ int32_t ack_vq_batch(const AckDevice* dev, const AckBuffer* b0, const AckBuffer*
  * and the nibble columns and split-k partials of onehot-mfma) comes from a
  * fixed 16 MiB device array that each GPU holds until the process ends, in
  * place of memory ack_vq would allocate. A plan needing more than 16 MiB of
- * it is refused with ACK_ERR_SIZE (a joint-mfma product runs on the general
- * kernel instead, which needs none). The array belongs to one device handle at a time: calls on
+ * it is refused with ACK_ERR_SIZE (a joint-mfma product whose transposed codes
+ * would need more, that is two operands of over 32 Mi codes with k > 256, runs on
+ * the general kernel instead, in the shader's order: the one case whose bits are
+ * not ack_vq's). The array belongs to one device handle at a time: calls on
  * one handle are ordered on its stream, and a call through another handle
  * of the same GPU is refused with ACK_ERR_DEVICE (the message names the
  * scratch) while the previous owner's enqueued noalloc work has not
- * finished; after ack_sync on that handle it proceeds. */
+ * finished; after ack_sync on that handle it proceeds. The general, gram-mfma
+ * and joint-mfma paths never take the array: their partial sums and transposed
+ * codes lie in 8 MiB that each handle holds from ack_open on, and where those do
+ * not suffice the blocks do without them, in the same order and bits, only slower.
+ * ack_vq does without them too when the GPU has no memory left for them. */
 int32_t ack_vq_noalloc(const AckDevice* dev, const AckBuffer* b0, const AckBuffer* b1,
                        const AckBuffer* b2, const AckBuffer* b3, const AckBuffer* out,
                        const AckBuffer* status, const uint8_t* plan, size_t plan_len);
