@@ -103,19 +103,21 @@ __device__ __forceinline__ int book_exponent(const float* book, uint32_t entries
   return e;
 }
 
-// The power of two each book is scaled by. Packed A: both books below 1, so
-// the sums stay below k whatever the magnitudes. Dense A: B's only where its
-// entries are so small that their last term would be subnormal, and then to
-// 2^-60, so that no sum can overflow where the product does not.
+// The power of two each book is scaled by: up to 2^-60 where its entries are so
+// small that their last terms would be subnormal, and packed A down by 2^8 where the
+// products come near FP32's end, which a sum of hi terms may pass by 2^-8 when the
+// product does not. Never by a book's largest entry: no code may use it, and those
+// that codes do use would lose their last terms.
 struct Shifts {
   int a, b;
 };
 template <bool AD>
 __device__ __forceinline__ Shifts book_shifts(const float* a_book, const float* b_book,
                                               uint32_t entries) {
-  const int eb = book_exponent(b_book, entries);
-  if constexpr (AD) return {0, eb < -60 ? -60 - eb : 0};
-  return {-book_exponent(a_book, entries), -eb};
+  const int eb = book_exponent(b_book, entries), sb = eb < -60 ? -60 - eb : 0;
+  if constexpr (AD) return {0, sb};
+  const int ea = book_exponent(a_book, entries);
+  return {ea < -60 ? -60 - ea : ea + eb > 100 ? -8 : 0, sb};
 }
 
 // A packed operand's book, scaled and split: planes for 16-byte copies along a

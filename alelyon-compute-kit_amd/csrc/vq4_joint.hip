@@ -138,6 +138,22 @@ __device__ __forceinline__ int book_exponent(const float* book) {
   return e;
 }
 
+// The power of two that brings the book's largest magnitude into [2^-61, 2^top):
+// almost always 0, seen without a reduction.
+template <int ENTRIES>
+__device__ __forceinline__ int book_scale(const float* book, int top) {
+  bool large = false, usual = false;
+#pragma unroll
+  for (int i = 0; i < ENTRIES / 64; ++i) {
+    const float v = fabsf(book[threadIdx.x % 64 + 64 * i]);
+    large |= v >= ldexpf(1.0f, top);
+    usual |= v >= 0x1p-61f;
+  }
+  if (!__any(large) && __any(usual)) return 0;
+  const int e = book_exponent<ENTRIES>(book);
+  return e > top ? top - e : e < -60 ? -60 - e : 0;
+}
+
 // One thread's share of a step's words, gathered from the codes: word `w` (8
 // inner indices from 128 step + 8 w) of the block's column `at`, zero past k.
 __device__ __forceinline__ uint32_t gather_word(const uint32_t* codes, uint32_t columns, uint32_t v,
@@ -176,12 +192,15 @@ __global__ __launch_bounds__(kJointThreads, 2) void k_joint_mfma(Operands o, uin
     const float* a_book = item_ptr<float>(o.in[1], o.stride[1], item);
     const float* b_book = item_ptr<float>(o.in[3], o.stride[3], item);
     float* out = reinterpret_cast<float*>(static_cast<char*>(o.out) + o.stride[4] * item);
-    // ---- the books as operands: A's scaled below 1 by a power of two (and by
-    // the 1/4 of the counts' unit), B's by its inverse, so that no partial sum
-    // can overflow where the product does not. Group 8 fills an instruction's
-    // 16 sides with two vectors: its second operand set holds the book in sides
-    // 8 to 15.
-    const int ea = book_exponent<16 * G>(a_book);
+    // ---- the books as operands (A's times the 1/4 of the counts' unit). Entries
+    // that no code uses, or that never meet, add exact zeros, so a book needs a scale
+    // only where its counted entries (up to 2^16 times 2^128) would overflow, or where
+    // all of it is so small that the sums might be subnormal; scaling by its largest
+    // entry otherwise loses or overflows others. Group 8 fills an instruction's 16
+    // sides with two vectors: its second operand set holds the book in sides 8 to 15.
+    const int sa = book_scale<16 * G>(a_book, 109);
+    const int sb = book_scale<16 * G>(b_book, 128);
+    const int up = -(sa + sb);
     bool bad = false;
     if (blockIdx.x == 0 && blockIdx.y == 0)
       for (uint32_t i = threadIdx.x; i < 16 * G; i += kJointThreads)
@@ -193,8 +212,8 @@ __global__ __launch_bounds__(kJointThreads, 2) void k_joint_mfma(Operands o, uin
       for (int r = 0; r < 4; ++r) {
         const bool in = G >= 16 || (l16 / 8 == uint32_t(b));
         const uint32_t at = (4 * q + r) * G + (G >= 16 ? 16 * b + l16 : l16 % 8);
-        ca[b][r] = in ? ldexpf(a_book[at], -ea - 2) : 0.0f;
-        cb[b][r] = in ? ldexpf(b_book[at], ea) : 0.0f;
+        ca[b][r] = in ? ldexpf(a_book[at], sa - 2) : 0.0f;
+        cb[b][r] = in ? ldexpf(b_book[at], sb) : 0.0f;
       }
 
     f32x4 h[IG][JG];
@@ -321,7 +340,10 @@ __global__ __launch_bounds__(kJointThreads, 2) void k_joint_mfma(Operands o, uin
           const uint32_t iv = ig0 + i + l16 / 8, jv = jg0 + j + q / 2;
           if (iv < va && jv < vb) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) check = fmaf(c[r], 0.0f, check);
+            for (int r = 0; r < 4; ++r) {
+              c[r] = ldexpf(c[r], up);
+              check = fmaf(c[r], 0.0f, check);
+            }
             *reinterpret_cast<f32x4*>(out + (uint64_t(iv) * 8 + l16 % 8) * n + uint64_t(jv) * 8 +
                                       4 * (q % 2)) = c;
           }
@@ -346,7 +368,10 @@ __global__ __launch_bounds__(kJointThreads, 2) void k_joint_mfma(Operands o, uin
                 c = __builtin_amdgcn_mfma_f32_16x16x4f32(cb[tb][r], t[r], c, 0, 0, 0);
               if (live) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) check = fmaf(c[r], 0.0f, check);
+                for (int r = 0; r < 4; ++r) {
+                  c[r] = ldexpf(c[r], up);
+                  check = fmaf(c[r], 0.0f, check);
+                }
                 *reinterpret_cast<f32x4*>(out + (uint64_t(ig0 + i) * G + 16 * sb + l16) * n +
                                           uint64_t(jg0 + j) * G + 16 * tb + 4 * q) = c;
               }
