@@ -410,11 +410,22 @@ constexpr uint32_t kDecodeQuads = 4;
 // ---- op 1: decode -------------------------------------------------------
 // out[i] = book[code(i / G)][i % G], a bit copy. Each lane writes 16-byte quads
 // (G is a multiple of 4, so a quad never straddles vectors). Bound by the
-// writes: with the codes of four quads loaded together and non-temporal stores,
-// 8192 x 8192 values at group 8 into buffers no cache holds take 47 us (5.7
-// TB/s; a fill of them 39) against 60 with one quad a turn and plain stores
-// (42 only where one 256 MiB output is rewritten in the Infinity Cache).
-template <int G>
+// writes: with the codes of four quads loaded together, 8192 x 8192 values at group
+// 8 into buffers that no cache holds take 46 us (5.9 TB/s; a fill of them 39)
+// against 60 with one quad a turn.
+//
+// DIRECT: stores past the Infinity Cache (256 MiB), or the caches before it. us,
+// direct against not, alone into fresh buffers / alone into one / followed by an
+// encode that reads them / the same over one buffer:
+//   32 MiB   6.9 / 6.8 / 17.4 / 25.1  against   8.5 /   7.9 / 17.8 / 27.3
+//   96 MiB    17 /  17 /   40 /   43  against    18 /    17 /   39 /   48
+//  128 MiB    23 /  22 /   52 /   55  against    24 /    22 /   50 /   59
+//  192 MiB    35 /  35 /   76 /   77  against    35 /    31 /   70 /   80
+//  256 MiB    48 /  48 /  100 /  101  against    47 /    41 /   95 /  101
+//  512 MiB    97 /  96 /  198 /  198  against   101 /   100 /  198 /  199
+// so the outputs between 160 and 256 MiB are stored through the caches.
+constexpr uint64_t kCachedFrom = uint64_t(160) << 20, kCachedTo = uint64_t(256) << 20;
+template <int G, bool DIRECT>
 __global__ __launch_bounds__(kThreads) void k_decode(Operands o, uint32_t m) {
   const uint32_t item = blockIdx.y;
   const uint32_t* codes = item_ptr<uint32_t>(o.in[0], o.stride[0], item);
@@ -440,8 +451,10 @@ __global__ __launch_bounds__(kThreads) void k_decode(Operands o, uint32_t m) {
       for (uint32_t i = 0; i < kDecodeQuads; ++i) {
         const uint32_t e = (q0 + i * kThreads) * 4;
         const u32x4 v = *reinterpret_cast<const u32x4*>(sbook + code[i] * G + e % G);
-        if (q0 + i * kThreads < quads)
-          __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(out + e));
+        if (q0 + i * kThreads < quads) {
+          if (DIRECT) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(out + e));
+          else *reinterpret_cast<u32x4*>(out + e) = v;
+        }
       }
     }
   } else {
@@ -1078,11 +1091,18 @@ hipError_t launch_encode(hipStream_t s, const Operands& o, uint32_t m, uint32_t 
   return hipGetLastError();
 }
 
+template <bool DIRECT>
+static void run_decode(hipStream_t s, const Operands& o, uint32_t m, uint32_t group, dim3 grid) {
+  if (group == 8) k_decode<8, DIRECT><<<grid, kThreads, 0, s>>>(o, m);
+  else if (group == 16) k_decode<16, DIRECT><<<grid, kThreads, 0, s>>>(o, m);
+  else k_decode<32, DIRECT><<<grid, kThreads, 0, s>>>(o, m);
+}
+
 hipError_t launch_decode(hipStream_t s, const Operands& o, uint32_t m, uint32_t group) {
   dim3 grid(grid_for((m + 3) / 4, kThreads * kDecodeQuads), o.count);
-  if (group == 8) k_decode<8><<<grid, kThreads, 0, s>>>(o, m);
-  else if (group == 16) k_decode<16><<<grid, kThreads, 0, s>>>(o, m);
-  else k_decode<32><<<grid, kThreads, 0, s>>>(o, m);
+  const uint64_t bytes = uint64_t(m) * 4 * o.count;
+  if (bytes > kCachedFrom && bytes <= kCachedTo) run_decode<false>(s, o, m, group, grid);
+  else run_decode<true>(s, o, m, group, grid);
   return hipGetLastError();
 }
 
