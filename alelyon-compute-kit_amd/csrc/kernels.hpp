@@ -31,7 +31,7 @@ enum class MatmulPath : int {
   General = 0,    // tiled, sequential FP32 per output: bit-identical to vq4.comp
   GemvRows = 1,   // 2 <= m <= 8, B groups along n: nibble bins, two rows per 64-bit atomic
   GemvTable = 2,  // B groups along k (B stored (n,k)): dot-product table, small m
-  GramMfma = 3,   // both operands grouped along k: one-hot x Gram table on fp16 MFMA
+  GramMfma = 3,   // both operands grouped along k: one-hot x Gram table on 6-bit MFMA
   // 4 is retired: row bins, an FP32 add per (row, nibble) through VGPR index
   // mode, served dense activations of large m before onehot-mfma took them
   GemvPairs = 5,  // m = 1, B groups along n: one atomic per byte into 256-way pair bins
@@ -97,9 +97,10 @@ constexpr uint32_t kOneHotMinRowsSmall = 8;   // from here when B holds >= 2^20 
 // Group 32 (half the one-hot columns of group 16) past gemv-direct's size, up
 // to kOneHotMaxWeights32: from 4 packed rows (4096 x 14336 19.4 us against 28.8
 // on gemv-rows, 8192 x 8192 20.7 against 29.7; 3 rows 19.6 against 26.2 and 20.5
-// against 27.3, but 2 rows 19.9 against 19.1) and 5 dense (27.1 against 34.0,
-// 28.3 against 34.8; 4 rows 27.0 against 26.6). On 8192 x 14336 the bins win
-// (dense, 8 rows: 48 against 54).
+// against 27.3, but 2 rows 19.9 against 19.1) and 5 dense (26.1 against 35.3; 8
+// rows 24.3 against 44.2). On 8192 x 14336 the bins won (dense, 8 rows: 48 against
+// 54, before the split by bits). At group 16 4 packed rows on 4096 x 14336 take 31
+// on the bins, 5 39.5, and 8 36 here.
 constexpr uint32_t kOneHotMinRows32 = 4, kOneHotMinRowsDense32 = 5;
 constexpr uint64_t kOneHotMaxWeights32 = uint64_t(1) << 26;
 constexpr uint32_t kOneHotMinRowsDense = 9;   // the same for dense activations

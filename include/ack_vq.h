@@ -337,6 +337,10 @@ int32_t ack_vq_path_name(const uint8_t* plan, size_t plan_len, char* out, size_t
 int32_t ack_vq_batch_path_name(const uint8_t* plan, size_t plan_len, uint32_t count, char* out,
                                size_t len);
 
+/* Both names above are those of the path alone. "general" is two kernels, told
+ * apart by the plan: in the shader's order and bit-identical to it for k below 160
+ * (24 from 2^22 multiply-adds, m n k of one instance) and under policy 1, bf16 terms
+ * on matrix cores past that. */
 /* Path policy for one device: 0 = automatic, 1 = the general tiled kernel,
  * in the shader's order, for every matmul (a second implementation to
  * cross-check fast paths),

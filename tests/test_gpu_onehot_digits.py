@@ -1,6 +1,7 @@
-"""onehot-mfma on six-bit digits (packed A on large grids, k a multiple of 32):
-rows around the 128-row blocks, an odd number of 32-element blocks of k, book
-entries of any magnitude."""
+"""onehot-mfma at sizes that the six-bit digits and the bf16 terms share between
+them (packed A, k a multiple of 32; test_gpu_onehot_spread.py has the line): rows
+around the 128-row blocks, an odd number of 32-element blocks of k, book entries of
+any magnitude."""
 from __future__ import annotations
 
 import numpy as np
